@@ -415,7 +415,10 @@ int sfa_grid_barrier_cost(int blocks, int threads, int rounds, int mode,
  * solver/sparsesolver.cpp:1002-1335) over any number of device-resident
  * matrices; each step advances every running solve by one phase in one set of
  * three kernel launches (a captured graph replays 32 steps at a time), so
- * solves of any size share each launch.  Solves can be submitted and
+ * solves of any size share each launch.  A solve of a small matrix (its two
+ * gathered vectors fit the LDS of one CU: at most 8,190 rows, 16,382 in
+ * FP32) runs in a workgroup of its own beside those steps, as many phases in
+ * a call as the call asks for steps.  Solves can be submitted and
  * collected between sfa_batch_run calls (continuous batching).
  *   SFA_BATCH_FP64:  FP64 throughout; stopping rule of the reference
  *                    (sqrt(z.r) < max(precision*||b||, 2^-26)).
@@ -502,7 +505,8 @@ int sfa_batch_collect(sfa_batch b, int slot, double* x, sfa_batch_info* info);
 int sfa_batch_memory(sfa_batch b, long long* bytes);
 
 /* Steps the engine has executed since the batch was created (each step runs
- * the current phase of every running solve: four kernels). */
+ * the current phase of every running solve but those of small matrices:
+ * four kernels).  A run in which only small matrices solve takes no steps. */
 int sfa_batch_steps(sfa_batch b, long long* steps);
 /* Runs `steps` engine steps with the kernels launched on their own between
  * HIP events and adds their summed times, in milliseconds, to ms[0] (the two

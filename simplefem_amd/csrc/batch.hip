@@ -37,6 +37,9 @@
 // no-op, so replays past the end change nothing.  Between replays the host
 // admits new slots and collects finished ones: a new slot is counted by the
 // next k_batch_fold and joins the schedule that k_batch_prefix builds.
+//
+// Slots of small matrices take no part in the steps: each runs in a workgroup
+// of its own (k_batch_solo), on a second stream.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,6 +51,8 @@
 #include <vector>
 
 #include "../../include/simplefem_amd.h"
+#include "block_host.hpp"
+#include "block_solve.hpp"
 #include "device_common.hpp"
 #include "host_common.hpp"
 #include "kernels.hpp"
@@ -96,6 +101,7 @@ struct BSlot {
     int mat;
     int kind, group;
     int units;          // units of the phase in the step being scheduled
+    int solo;           // run by a workgroup of its own (k_batch_solo), never scheduled
     int mixed;
     int cont;           // mixed: inner solves continue the previous direction
     int K, maxK, exit_reason, outer, max_outer, inner_total;
@@ -830,7 +836,7 @@ __global__ void __launch_bounds__(kUnitBlock) k_batch_fold(BArgs<T> a)
     const int s = blockIdx.x;
     if (s >= sc->nslots) return;
     BSlot<T>& S = a.slots[s];
-    if (S.mat < 0 || S.kind == PH_DONE) {
+    if (S.mat < 0 || S.kind == PH_DONE || S.solo) {
         if (threadIdx.x == 0) S.units = 0;
         return;
     }
@@ -992,6 +998,150 @@ __global__ void __launch_bounds__(kPrefixBlock) k_batch_prefix(BArgs<T> a)
     }
 }
 
+// One slot per workgroup: the slots of small matrices (Engine::solo_matrix),
+// listed in list[0..gridDim.x).  A lockstep step costs four launches, 15-20 us
+// however little it has to do, and a small system needs 10 to 60 of them per
+// iteration; its own workgroup runs an iteration in 9 to 40 us up to 4,096
+// rows (block_solve.hpp), 256 such slots at a time, and waits for no other
+// slot.  Four right-hand sides each of twelve 2D systems of 36 to 4,096 rows:
+// 61.5 -> 4.3 ms in FP64, 86 -> 4.8 ms in mixed precision.
+// Runs the slot's program, a restart or an iteration at a time, until it is
+// done or `budget` phases have run; the state then stands in the slot as
+// between two steps.
+template <typename T>
+__global__ void __launch_bounds__(kBlockThreads) k_batch_solo(BArgs<T> a,
+                                                              const BlockMatrix<T>* __restrict__ bms,
+                                                              const int* __restrict__ list,
+                                                              int budget)
+{
+    extern __shared__ __align__(16) char lds[];
+    __shared__ double red[2][kBlockWaves];
+    __shared__ BSlot<T> S;
+    __shared__ BlockScalars c;
+    const int s = list[blockIdx.x];
+    const int tid = threadIdx.x;
+    if (tid == 0) S = a.slots[s];
+    __syncthreads();
+    const int mat = __builtin_amdgcn_readfirstlane(S.mat);
+    const BMat<T>& M = a.mats[mat];
+    BlockMatrix<T> BM = bms[mat];
+    BM.cols = block_global(BM.cols);
+    BM.vals = block_global(BM.vals);
+    BM.rows = block_global(BM.rows);
+    BM.diag = block_global(BM.diag);
+    BM.list = block_global(BM.list);
+    BM.heads = block_global(BM.heads);
+    const int ls = __builtin_amdgcn_readfirstlane(S.ls);
+    T* const x = block_global(S.x);
+    T* const r = block_global(S.r);
+    T* const b = block_global(S.b);
+    T* const d = block_global(S.d);
+    const int n = BM.n, na = BM.n_active;
+    BlockSolver<T> B(BM, lds, red, x, r, ls);
+    B.load_lists();
+    auto load_direction = [&] {
+        for (int i = tid; i < block_vector(n); i += kBlockThreads)
+            B.di(i) = i < n ? d[(size_t)i * ls] : T(0);
+    };
+    auto store_direction = [&] {
+        for (int i = tid; i < na; i += kBlockThreads) d[(size_t)i * ls] = B.di(i);
+    };
+    load_direction();
+    __syncthreads();
+    int kind = __builtin_amdgcn_readfirstlane(S.kind);
+    while (kind != PH_DONE && budget > 0) {
+        if (kind == PH_RESID || kind == PH_SPMV) {
+            const bool restart = kind == PH_RESID;
+            const int K0 = restart ? 0 : __builtin_amdgcn_readfirstlane(S.K);
+            const int per = M.gf + M.gb + 2;  // phases of an iteration or a restart
+            if (tid == 0) {
+                c = BlockScalars{};
+                c.small_breaks = 1;
+                c.zr = c.zr_end = S.zr;  // the recursive z.r the last inner solve ended with
+                c.tol2 = S.tol2;
+                c.rel2 = S.rel2;
+                c.K = S.K;
+                c.maxK = S.maxK;
+                c.reason = S.exit_reason;
+                c.zr_cont = S.zr_cont;
+                c.k_cont = S.k_cont;
+            }
+            __syncthreads();
+            B.run(b, restart, restart ? budget / per : max(1, budget / per), c);
+            const int ran = __builtin_amdgcn_readfirstlane(c.K) - K0;
+            budget -= (ran + (restart ? 1 : 0)) * per;
+            if (tid == 0) {
+                S.zr = c.zr;
+                S.tol2 = c.tol2;
+                S.K = c.K;
+                S.maxK = c.maxK;
+                S.exit_reason = c.reason;
+                S.zr_cont = c.zr_cont;
+                S.alpha = c.alpha;
+                S.beta = c.beta;
+                S.dAd = c.dAd;
+                if (S.mixed) S.inner_total += ran;
+                S.kind = PH_SPMV, S.group = 0;
+                if (c.ended) {
+                    if (S.mixed && S.cont && c.reason == SFA_EXIT_CONVERGED && ran > 0 &&
+                        c.zr_prev > 0. && isfinite(c.zr_prev)) {
+                        S.zr_cont = c.zr_prev;
+                        S.k_cont = c.K;
+                    }
+                    finish_solve(S);
+                }
+            }
+        } else if (kind == PH_RES64) {
+            if constexpr (sizeof(T) == 4) {  // the LDS vectors make room for x in FP64
+                store_direction();
+                __syncthreads();
+                double* const xl = reinterpret_cast<double*>(lds);
+                const double* const x64 = block_global(S.x64);
+                const double* const b64 = block_global(S.b64);
+                double* const r64 = block_global(S.r64);
+                for (int i = tid; i <= n; i += kBlockThreads)
+                    xl[i] = i < n ? x64[(size_t)i * ls] : 0.;
+                __syncthreads();
+                const SellViewT<double> F = M.full64;
+                double part = 0.;
+                for (int j = B.wave; j < M.full_slices; j += kBlockWaves) {
+                    const int row = group_row(F, j, j, B.lane, M.full_row0, na);
+                    if (row >= 0) {
+                        const double acc = sell_row<true>(F, j, B.lane, xl, b64[(size_t)row * ls]);
+                        r64[(size_t)row * ls] = acc;
+                        part += acc * acc;
+                    }
+                }
+                const double total = B.sum(part);
+                load_direction();
+                if (tid == 0) phase_complete(S, M, total);
+            }
+            budget--;
+        } else {  // PH_CONVERT, PH_CORRECT
+            double* const x64 = block_global(S.x64);
+            const double* const r64 = block_global(S.r64);
+            for (int i = tid; i < na; i += kBlockThreads) {
+                if (kind == PH_CORRECT) {
+                    x64[(size_t)i * ls] += (double)x[(size_t)i * ls];
+                } else {
+                    b[(size_t)i * ls] = (T)r64[(size_t)i * ls];
+                    x[(size_t)i * ls] = T(0);
+                    r[(size_t)i * ls] = T(0);
+                }
+            }
+            __syncthreads();  // every thread has read S
+            if (tid == 0) phase_complete(S, M, 0.);
+            budget--;
+        }
+        __syncthreads();
+        kind = __builtin_amdgcn_readfirstlane(S.kind);
+        __syncthreads();
+    }
+    store_direction();
+    __syncthreads();
+    if (tid == 0) a.slots[s] = S;
+}
+
 // SpMV autotuning probe (nm <= kMaxSlots): the PH_SPMV units of the matrices mats[0..nm) with
 // K lanes per row, grid-stride as k_batch_step runs them (unit u belongs to
 // the matrix m with ustart[m] <= u < ustart[m+1]); d and q are scratch
@@ -1027,6 +1177,7 @@ __global__ void __launch_bounds__(kUnitBlock) k_batch_spmv_probe(const BMat<T>* 
 
 constexpr int kStepBlocks = 2048;  // grid of k_batch_step: 8 blocks of 256 threads per CU
 constexpr int kGraphSteps = 32;    // steps per replay of the captured graph
+constexpr int kSoloPhases = 1 << 17;  // most phases of one k_batch_solo launch: under a second
 
 template <typename T>
 struct HostMat {
@@ -1041,6 +1192,7 @@ struct HostMat {
     T* diag = nullptr;
     int max_units = 1, gb = 0;
     int slots_in_use = 0;
+    BlockLayout<T> solo;  // lds > 0: its slots run in a workgroup of their own
     int bucket = 0;   // SpMV row-length bucket of the matrix (its full part's main one)
     BMat<T> bm{};     // host copy of the device table entry
 
@@ -1055,6 +1207,7 @@ struct HostMat {
             dev_free(p);
         fslice = frow0 = frows = bslice = brow0 = brows = nullptr;
         diag = nullptr;
+        solo.release();
         live = false;
     }
 };
@@ -1116,7 +1269,10 @@ struct Engine {
     std::vector<SlotVectors<T>> vecs;
     std::vector<int> slot_used;
     BMat<T>* d_mats = nullptr;
+    BlockMatrix<T>* d_bms = nullptr;          // the same table for k_batch_solo
     int d_mats_cap = 0;
+    hipStream_t solo_stream = nullptr;        // k_batch_solo runs beside the lockstep steps
+    int* d_list = nullptr;                    // its slots
     BSlot<T>* d_slots = nullptr;
     BSched* d_sched = nullptr;
     BSched* h_sched = nullptr;                // pinned
@@ -1132,17 +1288,24 @@ struct Engine {
     void release()
     {
         if (stream) (void)hipStreamSynchronize(stream);
+        if (solo_stream) (void)hipStreamSynchronize(solo_stream);
         if (graph) (void)hipGraphExecDestroy(graph);
         graph = nullptr;
         graph_rec.reset();
         for (auto& v : vecs) v.release();
         for (auto& m : mats) m.release();
         dev_free(d_mats);
+        dev_free(d_bms);
+        dev_free(d_list);
         dev_free(d_slots);
         dev_free(d_sched);
         pinned_free(h_sched);
         if (stream) (void)hipStreamDestroy(stream);
+        if (solo_stream) (void)hipStreamDestroy(solo_stream);
+        solo_stream = nullptr;
         d_mats = nullptr;
+        d_bms = nullptr;
+        d_list = nullptr;
         d_slots = nullptr;
         d_sched = nullptr;
         h_sched = nullptr;
@@ -1159,6 +1322,8 @@ struct Engine {
         cont = mixed_ == 1;
         max_slots = max_slots_;
         SFA_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        SFA_HIP(hipStreamCreateWithFlags(&solo_stream, hipStreamNonBlocking));
+        d_list = dev_alloc<int>(max_slots);
         slots.assign(max_slots, BSlot<T>{});
         for (auto& sl : slots) {
             sl.mat = -1;
@@ -1258,17 +1423,25 @@ struct Engine {
         bm.omega = T(omega);
         bm.c2 = T((2. - omega) / omega);
         M.bm = bm;
-        if (id >= d_mats_cap) {  // grow the device table (no kernel is running)
+        M.solo.create(plan, M.full, M.lower, M.upper, M.diag, stream);
+        M.bytes += M.solo.bytes;
+        const BlockMatrix<T> sm = M.solo.M;
+        if (id >= d_mats_cap) {  // grow the device tables (no kernel is running)
             const int cap = std::max(16, 2 * d_mats_cap);
             BMat<T>* nm = dev_alloc<BMat<T>>(cap);
+            BlockMatrix<T>* ns = dev_alloc<BlockMatrix<T>>(cap);
             if (d_mats) {
                 SFA_HIP(hipMemcpy(nm, d_mats, sizeof(BMat<T>) * d_mats_cap, hipMemcpyDeviceToDevice));
+                SFA_HIP(hipMemcpy(ns, d_bms, sizeof(BlockMatrix<T>) * d_mats_cap, hipMemcpyDeviceToDevice));
                 dev_free(d_mats);
+                dev_free(d_bms);
             }
             d_mats = nm;
+            d_bms = ns;
             d_mats_cap = cap;
         }
         SFA_HIP(hipMemcpy(d_mats + id, &bm, sizeof(BMat<T>), hipMemcpyHostToDevice));
+        SFA_HIP(hipMemcpy(d_bms + id, &sm, sizeof(BlockMatrix<T>), hipMemcpyHostToDevice));
         return id;
     }
 
@@ -1526,6 +1699,7 @@ struct Engine {
             sl.maxK = n;
             sl.exit_reason = SFA_EXIT_CAP;
             sl.max_outer = max_outer;
+            sl.solo = M.solo.lds > 0 ? 1 : 0;
             sl.ls = nrhs;
             sl.lane = k;
             sl.vgroup = s0;
@@ -1608,22 +1782,70 @@ struct Engine {
         graph_wide = w;
     }
 
+    // The running slots with a workgroup of their own, the longest solves
+    // first; *others: whether any other slot is running.
+    std::vector<int> solo_slots(bool* others)
+    {
+        running();
+        std::vector<int> list;
+        *others = false;
+        for (int s = 0; s < max_slots; s++) {
+            if (!slot_used[s] || slots[s].kind == PH_DONE) continue;
+            if (slots[s].solo) list.push_back(s);
+            else *others = true;
+        }
+        std::stable_sort(list.begin(), list.end(), [&](int a, int b) {
+            return mats[slots[a].mat].full.stored > mats[slots[b].mat].full.stored;
+        });
+        return list;
+    }
+
+    // Queues k_batch_solo over the listed slots on stream s; every solve's
+    // uploads have been waited for (submit_group).
+    void launch_solo(const std::vector<int>& list, int budget, hipStream_t s)
+    {
+        size_t lds = 0;
+        for (int k : list) lds = std::max(lds, mats[slots[k].mat].solo.lds);
+        SFA_HIP(hipMemcpyAsync(d_list, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice, s));
+        SFA_HIP(launch_lds(k_batch_solo<T>, dim3((unsigned)list.size()), dim3(kBlockThreads), lds, s,
+                           args(), (const BlockMatrix<T>*)d_bms, (const int*)d_list, budget));
+    }
+
     // Runs about max_steps steps (whole graph replays, at least one; 0: until
-    // no solve is running).  Returns the number of solves still running.
+    // no solve is running).  Slots with a workgroup of their own run as many
+    // phases beside them, on a second stream; the two touch no common slot.
+    // Returns the number of solves still running.
     int run(int max_steps)
     {
         SFA_HIP(hipSetDevice(device));
         if (!d_mats) return running();
-        build_graph();
-        if (max_steps > 0) {
-            const int reps = std::max(1, max_steps / kGraphSteps);
-            for (int i = 0; i < reps; i++) SFA_HIP(hipGraphLaunch(graph, stream));
-        } else {
-            // the first replay also schedules slots admitted since the last one
-            do {
-                SFA_HIP(hipGraphLaunch(graph, stream));
-                read_sched();
-            } while (h_sched->active > 0);
+        bool others = false;
+        std::vector<int> solo = solo_slots(&others);
+        const int reps = max_steps > 0 ? std::max(1, max_steps / kGraphSteps) : 0;
+        try {
+            if (!solo.empty()) launch_solo(solo, max_steps > 0 ? reps * kGraphSteps : kSoloPhases, solo_stream);
+            if (others) {
+                build_graph();
+                if (max_steps > 0) {
+                    for (int i = 0; i < reps; i++) SFA_HIP(hipGraphLaunch(graph, stream));
+                } else {
+                    // the first replay also schedules slots admitted since the last one
+                    do {
+                        SFA_HIP(hipGraphLaunch(graph, stream));
+                        read_sched();
+                    } while (h_sched->active > 0);
+                }
+            }
+            SFA_HIP(hipStreamSynchronize(solo_stream));
+            while (max_steps == 0 && !solo.empty()) {  // solves longer than one launch's phases
+                bool none = false;
+                solo = solo_slots(&none);
+                if (!solo.empty()) launch_solo(solo, kSoloPhases, solo_stream);
+                SFA_HIP(hipStreamSynchronize(solo_stream));
+            }
+        } catch (...) {
+            (void)hipStreamSynchronize(solo_stream);
+            throw;
         }
         read_sched();
         return running();
@@ -1644,8 +1866,11 @@ struct Engine {
         };
         try {
             for (auto& e : ev) SFA_HIP(hipEventCreate(&e));
+            bool others = false;
+            const std::vector<int> solo = solo_slots(&others);
             for (int i = 0; i < steps; i++) {
                 SFA_HIP(hipEventRecord(ev[4 * i], stream));
+                if (i == 0 && !solo.empty()) launch_solo(solo, steps, stream);
                 launch_step(a, wide());
                 SFA_HIP(hipEventRecord(ev[4 * i + 1], stream));
                 launch(k_batch_fold<T>, dim3(max_slots), dim3(kUnitBlock), stream, a);

@@ -204,6 +204,18 @@ struct DevPartT {
 };
 using DevPart = DevPartT<double>;
 
+// Whether the first backward group holds the rows of the last forward group
+// and no entries (the last colour): its rows then need only their own m.
+template <typename T>
+bool first_backward_is_last_forward(const DevPartT<T>& lower, const DevPartT<T>& upper)
+{
+    if (lower.ngroups() == 0 || upper.ngroups() == 0) return false;
+    const int gl = lower.ngroups() - 1;
+    return lower.row0(gl) >= 0 && upper.row0(0) == lower.row0(gl) &&
+           upper.nrows_of(0) == lower.nrows_of(gl) &&
+           upper.group_count(0) == lower.group_count(gl) && upper.group_entries[0] == 0;
+}
+
 // Per-launch HIP events of a profiled solve.
 struct Profiler {
     std::vector<hipEvent_t> pool;

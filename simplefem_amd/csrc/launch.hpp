@@ -62,6 +62,21 @@ void fill_pointers(Tuple& t, void** ptrs, std::index_sequence<I...>)
 
 }  // namespace detail
 
+// A launch with `lds` bytes of dynamic LDS, never recorded; above 64 KiB the
+// kernel is first allowed that much (gfx950 has 160 KiB per CU).
+template <typename... P, typename... A>
+hipError_t launch_lds(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream,
+                      A&&... args)
+{
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    kernel<<<grid, block, lds, stream>>>(static_cast<P>(std::forward<A>(args))...);
+    return hipGetLastError();
+}
+
 template <typename... P, typename... A>
 void launch(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t stream, A&&... args)
 {

@@ -276,11 +276,7 @@ struct SystemT {
         }
         has_lower_restart = plan.has_lower_restart;
         if (sweeps && !eisen && lower.ngroups() > 0 && upper.ngroups() > 0) {
-            const int gl = lower.ngroups() - 1;
-            fuse_first_backward = lower.row0(gl) >= 0 && upper.row0(0) == lower.row0(gl) &&
-                                  upper.nrows_of(0) == lower.nrows_of(gl) &&
-                                  upper.group_count(0) == lower.group_count(gl) &&
-                                  upper.group_entries[0] == 0;
+            fuse_first_backward = first_backward_is_last_forward(lower, upper);
             // The first forward group (no lower entries) runs inside the second
             // one's kernel; its x, r updates move to its own backward kernel,
             // the last one, which must cover the same rows.
