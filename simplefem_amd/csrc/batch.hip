@@ -1009,13 +1009,14 @@ __global__ void __launch_bounds__(kPrefixBlock) k_batch_prefix(BArgs<T> a)
 // done or `budget` phases have run; the state then stands in the slot as
 // between two steps.
 template <typename T>
-__global__ void __launch_bounds__(kBlockThreads) k_batch_solo(BArgs<T> a,
+__global__ void __launch_bounds__(block_threads<T>) k_batch_solo(BArgs<T> a,
                                                               const BlockMatrix<T>* __restrict__ bms,
                                                               const int* __restrict__ list,
                                                               int budget)
 {
+    constexpr int kBlockThreads = block_threads<T>;
     extern __shared__ __align__(16) char lds[];
-    __shared__ double red[2][kBlockWaves];
+    __shared__ double red[2][kBlockMaxWaves];
     __shared__ BSlot<T> S;
     __shared__ BlockScalars c;
     const int s = list[blockIdx.x];
@@ -1029,6 +1030,7 @@ __global__ void __launch_bounds__(kBlockThreads) k_batch_solo(BArgs<T> a,
     BM.vals = block_global(BM.vals);
     BM.rows = block_global(BM.rows);
     BM.diag = block_global(BM.diag);
+    BM.precon = nullptr;
     BM.list = block_global(BM.list);
     BM.heads = block_global(BM.heads);
     const int ls = __builtin_amdgcn_readfirstlane(S.ls);
@@ -1104,7 +1106,7 @@ __global__ void __launch_bounds__(kBlockThreads) k_batch_solo(BArgs<T> a,
                 __syncthreads();
                 const SellViewT<double> F = M.full64;
                 double part = 0.;
-                for (int j = B.wave; j < M.full_slices; j += kBlockWaves) {
+                for (int j = B.wave; j < M.full_slices; j += block_waves<T>) {
                     const int row = group_row(F, j, j, B.lane, M.full_row0, na);
                     if (row >= 0) {
                         const double acc = sell_row<true>(F, j, B.lane, xl, b64[(size_t)row * ls]);
@@ -1807,7 +1809,7 @@ struct Engine {
         size_t lds = 0;
         for (int k : list) lds = std::max(lds, mats[slots[k].mat].solo.lds);
         SFA_HIP(hipMemcpyAsync(d_list, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice, s));
-        SFA_HIP(launch_lds(k_batch_solo<T>, dim3((unsigned)list.size()), dim3(kBlockThreads), lds, s,
+        SFA_HIP(launch_lds(k_batch_solo<T>, dim3((unsigned)list.size()), dim3(dev::block_threads<T>), lds, s,
                            args(), (const BlockMatrix<T>*)d_bms, (const int*)d_list, budget));
     }
 

@@ -13,6 +13,15 @@ namespace sfa {
 
 constexpr size_t kBlockMaxLds = 150 * 1024;  // of a CU's 160 KiB
 
+// The loop of a solve in one workgroup (block.hip): the restart, when asked
+// for, and at most max_iters iterations; zr_cont > 0: the restart continues
+// the direction dprev (see BlockScalars).
+template <typename T>
+hipError_t launch_block_solve(hipStream_t s, const dev::BlockMatrix<T>& M, size_t lds,
+                              SolveState* st, T* x, T* r, const T* b, T* d, T* d1, int restart,
+                              int max_iters, double zr_cont, double zr_end, int k_cont,
+                              const T* dprev);
+
 // A system in the layout of one workgroup; lds 0: it does not fit.
 template <typename T>
 struct BlockLayout {
@@ -43,6 +52,7 @@ struct BlockLayout {
                 const DevPartT<T>& upper, const T* device_diag, hipStream_t s)
     {
         using namespace dev;
+        constexpr int kBlockWaves = block_waves<T>;
         release();
         const int n = plan.n;
         if ((size_t)block_vector(n) * sizeof(T) > 65536) return;
@@ -75,8 +85,8 @@ struct BlockLayout {
         auto even = [&](int w, size_t from) {
             if ((lists[w].size() - from) % 2) lists[w].insert(lists[w].begin() + from, make_uint2(0u, 0u));
         };
-        const int gl = plan.lower.ngroups(), gu = plan.upper.ngroups();
-        const int back = gu - (fuse ? 1 : 0);
+        const int gl = std::max(0, plan.lower.ngroups()), gu = std::max(0, plan.upper.ngroups());
+        const int back = gu - (fuse ? 1 : 0);  // CG and Jacobi: no groups
         for (int g = 0; g < gl; g++)
             phase(plan.lower, 0, g, (fuse && g == gl - 1 ? kItemFused : 0u) |
                                         (g == gl - 1 && back == 0 ? kItemSwept : 0u));
@@ -101,6 +111,7 @@ struct BlockLayout {
         const size_t ns = slices.size(), lanes = std::max<size_t>(ns, 1) * kSliceRows,
                      entries = std::max<size_t>(chunks, 1) * kSliceRows;
         M.sweeps = gl + back > 0 ? 1 : 0;
+        M.precon = plan.method == SFA_METHOD_DIAGONAL ? device_diag : nullptr;
         M.n = n;
         M.n_active = plan.n_active;
         M.omega = T(plan.omega);

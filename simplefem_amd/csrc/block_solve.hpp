@@ -1,9 +1,9 @@
-// block_solve.hpp -- the CG-SSOR loop of a small system inside one workgroup.
+// block_solve.hpp -- the CG loop of a small system inside one workgroup.
 //
 // A launch per colour costs 3.6-3.9 us whatever its size (half of it the
 // kernel boundary), so a system of a few thousand rows spends all its time
-// on launches: 57 us per iteration for a 33^2 P1 mesh whose data one CU
-// reads in 2 us.  Here one 1024-thread workgroup runs the loop, a workgroup
+// on launches: 53 us per iteration for a 33^2 P1 mesh whose data one CU
+// reads in 2 us.  Here one workgroup runs the loop, a workgroup
 // barrier between colours.  What bounds it then is the chain of a colour --
 // gather, sum, division, barrier, about 0.2 us -- and every instruction
 // beside it, so the layout takes work off that chain:
@@ -30,11 +30,18 @@
 namespace sfa {
 namespace dev {
 
-// 16 wavefronts: with 4 (8) the 48 solves of twelve 2D systems of 36 to 4,096
-// rows take 6.1 ms (4.5) instead of 4.3, a system alone up to 4,096 rows 48 us
-// (36) per iteration instead of 34, and up to 1,000 rows the same.
-constexpr int kBlockWaves = 16;
-constexpr int kBlockThreads = kBlockWaves * kWave;
+// Wavefronts of the workgroup.  Every wavefront runs the scalar steps and walks
+// its list at 4 cycles an instruction, so more of them cost more where there
+// are few slices to share, and the registers of 16 do not hold two FP64 slices
+// in flight: 4 / 8 / 16 wavefronts take 6.1 / 4.5 / 4.3 ms for the 48 FP64
+// solves of twelve 2D systems of 36 to 4,096 rows, 8 / 16 take 0.55 / 0.75 ms
+// for one SSOR solve of a 33^2 mesh, and in FP32 5.5 / 4.8 ms and 7.2 / 5.8 ms
+// for those twelve systems and an H(curl) system of 5,859 rows.
+template <typename T>
+constexpr int block_waves = sizeof(T) == 8 ? 8 : 16;
+template <typename T>
+constexpr int block_threads = block_waves<T> * kWave;
+constexpr int kBlockMaxWaves = 16;
 constexpr int kBlockChunk = 4;       // entries per lane and chunk
 
 // A wavefront's slice of a phase, as its list holds it: .x the slice's first
@@ -59,7 +66,8 @@ struct BlockMatrix {
     const int* heads;            // wavefront w's from heads[w] to heads[w + 1], the
                                  // product's from heads[kBlockWaves + 1 + w]
     int list_size, r_in_lds;
-    int sweeps;                  // 0: no active rows
+    const T* precon;             // device order; CG without sweeps: z = precon r, or null: z = r
+    int sweeps;                  // 1: z comes from the sweeps
     int n, n_active;
     T omega, c2;
 };
@@ -140,7 +148,8 @@ __device__ inline double dpp_wave_sum(double v)
 
 template <typename T>
 struct BlockSolver {
-    static constexpr int NC = 2;  // chunks of an item held in registers
+    static constexpr int kBlockWaves = block_waves<T>, kBlockThreads = block_threads<T>;
+    static constexpr unsigned NC = 2;  // chunks of an item held in registers
     struct Item {
         unsigned at, what;  // its list entry
         uint2 c[NC];
@@ -153,7 +162,7 @@ struct BlockSolver {
     char* w;         // LDS: block_vector(n) entries, entry n 0
     char* dl;        // LDS: the direction, likewise
     T* rl;           // LDS: r, or null
-    double (*red)[kBlockWaves];  // LDS [2]
+    double (*red)[kBlockMaxWaves];  // LDS [2]
     uint2* items;    // LDS: every wavefront's list
     T *x, *r;        // element i at v[i * ls]
     int ls;
@@ -171,7 +180,7 @@ struct BlockSolver {
         return ((size_t)2 * block_vector(n) * sizeof(T) + 15) / 16 * 16;
     }
 
-    __device__ BlockSolver(const BlockMatrix<T>& M_, char* lds, double (*red_)[kBlockWaves], T* x_,
+    __device__ BlockSolver(const BlockMatrix<T>& M_, char* lds, double (*red_)[kBlockMaxWaves], T* x_,
                            T* r_, int ls_)
         : M(M_), red(red_), x(x_), r(r_), ls(ls_)
     {
@@ -198,15 +207,35 @@ struct BlockSolver {
         for (int i = tid; i < M.list_size; i += kBlockThreads) items[i] = M.list[i];
     }
 
-    // fn(i, ri) for the rows this thread owns, ri a reference to r_i.
-    template <class Fn>
-    __device__ void own_rows(Fn&& fn)
+    // fn(i, v_i) for the rows this thread owns, four of a vector's loads in
+    // flight; STORE: fn's result is stored back.  v has stride `stride`.
+    template <bool STORE, class Fn>
+    __device__ void own_rows(T* v, int stride, Fn&& fn) const
     {
-        if (rl) {
-            for (int i = tid; i < M.n_active; i += kBlockThreads) fn(i, rl[i]);
-        } else {
-            for (int i = tid; i < M.n_active; i += kBlockThreads) fn(i, at(r, i));
+        constexpr int U = 4;
+        for (int i0 = tid; i0 < M.n_active; i0 += U * kBlockThreads) {
+            T t[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = i0 + u * kBlockThreads;
+                t[u] = v[(size_t)(i < M.n_active ? i : i0) * stride];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = i0 + u * kBlockThreads;
+                if (i < M.n_active) {
+                    if constexpr (STORE) v[(size_t)i * stride] = fn(i, t[u]);
+                    else fn(i, t[u]);
+                }
+            }
         }
+    }
+    // The same over r, wherever it lives.
+    template <bool STORE, class Fn>
+    __device__ void own_r(Fn&& fn) const
+    {
+        if (rl) own_rows<STORE>(rl, 1, fn);
+        else own_rows<STORE>(r, ls, fn);
     }
 
     // Sum over the workgroup in a fixed order; every thread gets the same
@@ -259,8 +288,8 @@ struct BlockSolver {
         I.row = M.rows[slot];
         I.dg = M.diag[slot];
 #pragma unroll
-        for (int k = 0; k < NC; k++) {
-            if ((unsigned)k < nc) {
+        for (unsigned k = 0; k < NC; k++) {
+            if (k < nc) {
                 I.c[k] = M.cols[(I.at + k) * kWave + (unsigned)lane];
                 load_values(I.at + k, I.v[k]);
             }
@@ -322,16 +351,16 @@ struct BlockSolver {
     __device__ T finish(const Item& I, char* vec, T acc) const
     {
         const unsigned nc = __builtin_amdgcn_readfirstlane(I.what) & (kItemMaxChunks - 1);
-        if (nc <= 2) {
-            if (nc == 1) return apply_chunk(acc, I.c[0], I.v[0], vec);
-            if (nc == 2) return apply_chunks(acc, I.c[0], I.v[0], I.c[1], I.v[1], vec);
-            return acc;
-        }
         const unsigned at = __builtin_amdgcn_readfirstlane(I.at);
         Pair A, B;
-        load_pair(A, at, 2, nc);
-        acc = apply_chunks(acc, I.c[0], I.v[0], I.c[1], I.v[1], vec);
-        for (unsigned k = 2;;) {
+        if (nc > NC) load_pair(A, at, NC, nc);
+#pragma unroll
+        for (unsigned k = 0; k < NC; k += 2) {
+            if (k + 1 < nc) acc = apply_chunks(acc, I.c[k], I.v[k], I.c[k + 1], I.v[k + 1], vec);
+            else if (k < nc) acc = apply_chunk(acc, I.c[k], I.v[k], vec);
+        }
+        if (nc <= NC) return acc;
+        for (unsigned k = NC;;) {
             load_pair(B, at, k + 2, nc);
             acc = apply_pair(acc, A, k, nc, vec);
             if ((k += 2) >= nc) return acc;
@@ -410,12 +439,12 @@ struct BlockSolver {
             for (int i = tid; i < block_vector(M.n); i += kBlockThreads) wi(i) = T(0);
         }
         if (rl)
-            for (int i = tid; i < M.n_active; i += kBlockThreads) rl[i] = at(r, i);
+            own_rows<false>(r, ls, [&](int i, T ri) { rl[i] = ri; });
         __syncthreads();
 
         auto residual_dot = [&]() -> double {
             double t = 0.;
-            own_rows([&](int i, T& ri) { t += (double)(wi(i) * ri); });
+            own_r<false>([&](int i, T ri) { t += (double)(wi(i) * ri); });
             return sum(t);
         };
         // The end of the restart's sweeps, at z.r: the first loop-head test
@@ -464,10 +493,10 @@ struct BlockSolver {
             }
             if (stop) return false;
             alpha = uniform((T)a);
-            own_rows([&](int i, T& ri) {
+            own_r<true>([&](int i, T ri) {
                 const T rr = ri - alpha * wi(i);
-                ri = rr;
                 wi(i) = rr;
+                return rr;
             });
             __syncthreads();
             return true;
@@ -475,13 +504,6 @@ struct BlockSolver {
         // The end of the sweeps: z.r, beta, K, the exit tests (:1299-1307), x
         // and d.
         auto swept = [&]() -> bool {
-            constexpr int X = 4;  // x values loaded ahead of the sum
-            T xk[X];
-#pragma unroll
-            for (int k = 0; k < X; k++) {
-                const int i = tid + k * kBlockThreads;
-                xk[k] = at(x, i < M.n_active ? i : 0);
-            }
             const double t = residual_dot();
             const double beta = t / zr;
             const double before = zr;
@@ -490,17 +512,11 @@ struct BlockSolver {
             max_iters--;
             const bool cap = K >= maxK;
             const bool ended = cap || ref_absolute(t) < tol2;
-            auto row = [&](int i, T xx) {
+            own_rows<true>(x, ls, [&](int i, T xx) {
                 const T dd = di(i);
-                at(x, i) = xx + alpha * dd;
                 if (!ended) di(i) = wi(i) + (T)beta * dd;
-            };
-#pragma unroll
-            for (int k = 0; k < X; k++) {
-                const int i = tid + k * kBlockThreads;
-                if (i < M.n_active) row(i, xk[k]);
-            }
-            for (int i = tid + X * kBlockThreads; i < M.n_active; i += kBlockThreads) row(i, at(x, i));
+                return xx + alpha * dd;
+            });
             __syncthreads();
             if (tid == 0) {
                 if (hist) hist[K] = t;
@@ -514,18 +530,17 @@ struct BlockSolver {
             return !ended && max_iters > 0;
         };
 
-        if (!M.sweeps) {  // no active rows: every sum is 0
-            bool on = restart ? restarted() && max_iters > 0 : max_iters > 0;
-            while (on) on = multiplied(0.) && swept();
-        } else if (restart || max_iters > 0) {
+        if (restart || max_iters > 0) {
             Item P, Q;
             bool starting = restart;
-            seek(restart ? first : product);
+            seek(restart ? first : product);  // without sweeps the two are one
             fetch(P);
             fetch(Q);
             for (bool skip = !restart;; skip = false) {
                 if (!skip) {
-                    for (;;) {  // the sweeps: a barrier between phases
+                    if (!M.sweeps)
+                        own_r<false>([&](int i, T ri) { wi(i) = M.precon ? M.precon[i] * ri : ri; });
+                    while (M.sweeps) {  // a barrier between phases
                         sweep(P);
                         const unsigned p = __builtin_amdgcn_readfirstlane(P.what);
                         fetch(P);

@@ -209,7 +209,7 @@ using DevPart = DevPartT<double>;
 template <typename T>
 bool first_backward_is_last_forward(const DevPartT<T>& lower, const DevPartT<T>& upper)
 {
-    if (lower.ngroups() == 0 || upper.ngroups() == 0) return false;
+    if (lower.ngroups() <= 0 || upper.ngroups() <= 0) return false;
     const int gl = lower.ngroups() - 1;
     return lower.row0(gl) >= 0 && upper.row0(0) == lower.row0(gl) &&
            upper.nrows_of(0) == lower.nrows_of(gl) &&

@@ -53,7 +53,7 @@ struct SolveState {
     int K;              // iterations done
     int done;           // 1 once the loop has ended
     int exit_reason;    // SFA_EXIT_*
-    int pad_;
+    int continued;      // 1: the restart continued an earlier direction (one-workgroup solves)
     double* hist;       // z.r at the top of iteration k, k = 0..K
 };
 

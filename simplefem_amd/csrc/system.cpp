@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/simplefem_amd.h"
+#include "block_host.hpp"
 #include "host_common.hpp"
 #include "kernels.hpp"
 #include "launch.hpp"
@@ -126,6 +127,19 @@ struct SystemT {
     std::unique_ptr<GraphRecorder> chunk_graph;  // the recorded graph and its arguments, kept with the exec
     int chunk_iters = 0;
     Profiler* prof = nullptr;  // set only while sfa_system_profile runs
+    bool launches = false;     // sfa_system_time_sweeps: the launch-by-launch path
+    // Small systems (not the Eisenstat variants): the loop in one workgroup.
+    // With sweeps, every system that fits; plain and Jacobi CG, two launches
+    // per iteration, only while one CU reads the matrix faster than those
+    // (us per iteration, launches -> one workgroup: 289 rows 15.8 -> 3.9,
+    // 4,225 rows and 29,057 entries 12.3 -> 8.6, 7,921 rows and 54,737
+    // entries 12.3 -> 15.3, 6,859 rows and 94,447 entries 15.2 -> 23.9; SSOR
+    // 33^2 52.8 -> 10.5, Rainbow 7,921 rows, 5 colours 34.4 -> 28.1, 6,859
+    // rows, 29 colours, 299,971 entries 572 -> 215).
+    BlockLayout<T> block;
+    static constexpr long long kBlockRowEntries = 40000;
+    static constexpr int kBlockIters = 4096;  // most iterations of one such launch
+    bool in_block() const { return block.lds > 0 && !prof && !launches; }
     // FP32 copy of the plan for the mixed-precision solve (T = double only)
     std::unique_ptr<SystemT<float>> inner;
 
@@ -161,6 +175,7 @@ struct SystemT {
         upper.release();
         lower_restart.release();
         apply_part.release();
+        block.release();
         if (!shares_perm) dev_free(perm);
         shares_perm = false;
         for (void* p : {(void*)diag, (void*)x, (void*)r, (void*)b, (void*)d, (void*)d1,
@@ -302,6 +317,9 @@ struct SystemT {
         std::vector<T> dg(plan.diag.begin(), plan.diag.end());
         dg.push_back(T(0));
         SFA_HIP(hipMemcpy(diag, dg.data(), (n + 1) * sizeof(T), hipMemcpyHostToDevice));
+
+        if (!eisen && (sweeps || full.stored <= kBlockRowEntries))
+            block.create(plan, full, lower, upper, diag, own_stream);
 
         T** vecs[] = {&x, &r, &b, &d, &d1, &z, &q, &m};
         for (T** v : vecs) {
@@ -749,15 +767,22 @@ struct SystemT {
         return s;
     }
 
-    // State, scratch and restart for x, b, r already in device order.
+    // State, scratch and restart for x, b, r already in device order (in one
+    // workgroup, the iterations as well).  zr_cont > 0: a solve in one workgroup
+    // may continue the direction in dkeep (solve_mixed).
     void start(hipStream_t s, double precision, int print_modulo, double host_tol,
-               int use_host_tol, double rel2, const T* rows_b = nullptr)
+               int use_host_tol, double rel2, const T* rows_b = nullptr, double zr_cont = 0.,
+               double zr_end = 0., int k_cont = 0)
     {
-        init_scratch(s);
         const int small_breaks = (method == SFA_METHOD_SSOR_EISENSTAT) ? (print_modulo >= -2) : 1;
+        if (!in_block()) init_scratch(s);
         launch_init_state(s, state, b, n, precision, host_tol, use_host_tol, n, small_breaks,
                           rel2, ps, rows_b);
-        restart(s);
+        if (in_block())
+            SFA_HIP(launch_block_solve<T>(s, block.M, block.lds, state, x, r, b, d, d1, 1, kBlockIters,
+                                          zr_cont, zr_end, k_cont, dkeep));
+        else
+            restart(s);
         read_state();
     }
 
@@ -797,6 +822,12 @@ struct SystemT {
     // Runs iterations until the state says the loop has ended.
     void iterate(hipStream_t s)
     {
+        while (in_block() && !host_state->done) {
+            SFA_HIP(launch_block_solve<T>(s, block.M, block.lds, state, x, r, b, d, d1, 0, kBlockIters,
+                                          0., 0., 0, (const T*)nullptr));
+            read_state();
+        }
+        if (host_state->done) return;
         // Iterations: replay a captured chunk, predicting from the z.r history
         // how many chunks to queue before the next look at the state.
         const int G = 4;
@@ -856,7 +887,14 @@ struct SystemT {
         SFA_HIP(hipSetDevice(device));
         hipStream_t s = stream;
         launch_fill(s, x, T(0), n);
-        start(s, 1e-10, -3, 0., 0, 0.);
+        launches = true;
+        try {
+            start(s, 1e-10, -3, 0., 0, 0.);
+        } catch (...) {
+            launches = false;
+            throw;
+        }
+        launches = false;
         if (host_state->done) throw Error{SFA_ERR_INVALID, "the restart already converged"};
         iteration(s, 0);
         const size_t per = klass == SFA_KERNEL_FORWARD ? fwd_sched.size() : bwd_sched.size();
@@ -1045,12 +1083,14 @@ struct SystemT {
                 SFA_HIP(hipMemcpyAsync(inner->dkeep, dlast, n * sizeof(float),
                                        hipMemcpyDeviceToDevice, s));
             }
-            inner->start(s, 1.0, -3, 0., 0, inner_rtol * inner_rtol);
+            inner->start(s, 1.0, -3, 0., 0, inner_rtol * inner_rtol, nullptr, zr_prev, zr_end, k_end);
             // Continue only where the FP64 residual agrees with the recursive
             // one the last inner solve ended with: a drifted FP32 residual
             // makes the old direction unfit (beta far too large).
-            if (zr_prev > 0. && !inner->host_state->done &&
-                inner->host_state->zr <= kContinueGap * zr_end) {
+            if (inner->in_block()) {
+                continued += inner->host_state->continued;
+            } else if (zr_prev > 0. && !inner->host_state->done &&
+                       inner->host_state->zr <= kContinueGap * zr_end) {
                 launch_direction_continue(s, inner->state, inner->n_active, inner->d,
                                           (const float*)inner->dkeep, zr_prev,
                                           (int)std::min<long long>(inner->n, std::max(100LL, 3LL * k_end)));

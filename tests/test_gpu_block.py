@@ -1,9 +1,9 @@
-"""Small systems run in one workgroup (csrc/block_solve.hpp): batch slots whose
-two gathered vectors fit a CU's LDS.
+"""Small systems run in one workgroup (csrc/block_solve.hpp): Systems and batch
+slots whose two gathered vectors fit a CU's LDS.
 
-The bars are those of the batch engine: K within max(1, 2%) of the oracle's,
-the same exit reason, x within 1e-10 relative; and a run cut into pieces gives
-the bits of one run.
+The bars are those of the solvers: K within max(1, 2%) of the oracle's, the
+same exit reason, x within 1e-10 relative; and a run cut into pieces gives the
+bits of one run.
 """
 import numpy as np
 import pytest
@@ -108,3 +108,85 @@ def test_batch_slot_breakdown_and_nan():
         assert info["exit_reason"] == capi.EXIT_BREAKDOWN and not info["success"]
         x, info = batch.collect(slots[1], s.n)
         _check(s, good, col, x, info)
+
+
+METHODS = {"cg": capi.METHOD_CG, "jacobi": capi.METHOD_DIAGONAL, "ssor": capi.METHOD_SSOR,
+           "rainbow": capi.METHOD_RAINBOW}
+
+
+def _solve(variant, s, b, x0=None, r0=None, omega=1.2, precision=1e-10):
+    """(system's, oracle's) x, residual and info of one solve."""
+    col = oracle.rainbow(s.n, s.A, s.C) if variant == "rainbow" else (0, None, None, None)
+    d = s.diagonal()
+    aux = {"cg": None, "jacobi": np.divide(1.0, d, out=np.zeros(s.n), where=d != 0)}.get(variant, d)
+    x = np.zeros(s.n) if x0 is None else x0.copy()
+    r = np.zeros(s.n) if r0 is None else r0.copy()
+    info = {}
+    with capi.System(METHODS[variant], s.n, s.A, s.C, s.V, aux, omega, *col) as system:
+        system.solve(x, b, r, precision, info=info)
+    want = oracle.solve(variant, s.A, s.C, s.V, b, x0=x0, residual0=r0, precision=precision,
+                        aux=aux, omega=omega, colouring=col if variant == "rainbow" else None)
+    return (x, r, info), want
+
+
+@pytest.mark.parametrize("variant", sorted(METHODS))
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_system_matches_oracle(name, variant):
+    """Nonzero x0 and residual0: rows a variant skips keep theirs."""
+    s = CASES[name]()
+    rng = np.random.default_rng(5)
+    b, x0, r0 = (rng.uniform(-1, 1, s.n) for _ in range(3))
+    b[s.diagonal() == 0] = 0.0
+    print(f"case: {variant} {name} n={s.n} nnz={s.nnz}", flush=True)
+    (x, r, info), (xo, ro, io) = _solve(variant, s, b, x0, r0)
+    assert abs(info["iterations"] - io["iterations"]) <= max(1, int(0.02 * io["iterations"])), (info, io)
+    assert info["exit_reason"] == io["exit_reason"], (info, io)
+    bad = np.isnan(xo)
+    assert np.array_equal(np.isnan(x), bad) and np.array_equal(np.isnan(r), np.isnan(ro))
+    if bad.any():
+        return
+    assert np.abs(x - xo).max() <= 1e-10 * max(np.abs(xo).max(), 1e-300)
+    # The loop may end an iteration earlier or later than the oracle's, so the
+    # residual is held against its own x: the recurrence drifts from b - A x by
+    # rounding only, a few hundred units in the last place of |A||x|.
+    true = b - oracle.csr_apply(s.n, s.A, s.C, s.V, x)
+    size = oracle.csr_apply(s.n, s.A, s.C, np.abs(s.V), np.abs(x)) + np.abs(b)
+    kept = (s.diagonal() == 0) & (variant != "cg")
+    assert np.array_equal(r[kept], r0[kept]) and np.array_equal(x[kept], x0[kept])
+    assert np.abs(r - true)[~kept].max(initial=0.0) <= 1e-13 * max(size.max(initial=0.0), 1e-300)
+
+
+def test_many_iterations_take_several_launches():
+    """One launch runs at most 4,096 iterations.  CG on the 1D Laplacian of
+    8,000 rows needs about as many as there are rows; its condition number is
+    2.6e7, so two FP64 solves agree to some 1e-8 and no better."""
+    n = 8000
+    rows = np.repeat(np.arange(n), 3)
+    cols = rows + np.tile([-1, 0, 1], n)
+    vals = np.tile([-1.0, 2.0, -1.0], n)
+    keep = (cols >= 0) & (cols < n)
+    A = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=n))]).astype(np.int32)
+    s = S.CSRSystem("laplace1d", n, A, cols[keep].astype(np.int32), vals[keep], np.zeros(n, dtype=bool))
+    b = S.uniform_pm1(7, n)
+    (x, _, info), (xo, _, io) = _solve("cg", s, b, precision=1e-9)
+    print(f"case: 1D Laplacian, K {info['iterations']} oracle {io['iterations']}", flush=True)
+    assert io["iterations"] > 4096
+    assert info["exit_reason"] == io["exit_reason"]
+    assert abs(info["iterations"] - io["iterations"]) <= 0.02 * io["iterations"]
+    assert np.linalg.norm(x - xo) <= 1e-7 * np.linalg.norm(xo)
+
+
+def test_mixed_solve_continues_directions():
+    """The FP32 inner solves in one workgroup: the FP64 residual target is met,
+    and inner solves continue the previous one's direction."""
+    s = S.poisson3d_p1_kuhn(16)
+    b = S.rhs_uniform(s, 9)
+    col = oracle.rainbow(s.n, s.A, s.C)
+    with capi.System(capi.METHOD_RAINBOW, s.n, s.A, s.C, s.V, s.diagonal(), 1.0, *col,
+                     fp32_inner=True) as system:
+        x = np.zeros(s.n)
+        info = system.solve_mixed(x, b, 1e-10, inner_rtol=1e-2)
+    res = b - oracle.csr_apply(s.n, s.A, s.C, s.V, x)
+    res[s.dirichlet] = 0.0
+    assert info["success"] and np.linalg.norm(res) <= 1.0000001e-10 * np.linalg.norm(b)
+    assert info["outer"] >= 3 and 1 <= info["continued"] < info["outer"]
