@@ -32,6 +32,7 @@ DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-p
 SOURCES = [  # (source, compile as HIP)
     ("kernels.hip", True),
     ("block.hip", True),
+    ("team.hip", True),
     ("batch.hip", True),
     ("hodge.hip", True),
     ("noalloc.hip", True),

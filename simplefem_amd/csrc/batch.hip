@@ -58,6 +58,7 @@
 #include "kernels.hpp"
 #include "launch.hpp"
 #include "plan.hpp"
+#include "team.hpp"
 
 namespace sfa {
 namespace {
@@ -1821,6 +1822,7 @@ struct Engine {
     {
         SFA_HIP(hipSetDevice(device));
         if (!d_mats) return running();
+        SolveGuard guard(device);
         bool others = false;
         std::vector<int> solo = solo_slots(&others);
         const int reps = max_steps > 0 ? std::max(1, max_steps / kGraphSteps) : 0;

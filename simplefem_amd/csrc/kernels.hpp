@@ -54,6 +54,8 @@ struct SolveState {
     int done;           // 1 once the loop has ended
     int exit_reason;    // SFA_EXIT_*
     int continued;      // 1: the restart continued an earlier direction (one-workgroup solves)
+    int team_lost;      // 1: a launch by a team of workgroups gave up (team.hip)
+    int pad_;
     double* hist;       // z.r at the top of iteration k, k = 0..K
 };
 

@@ -26,6 +26,7 @@
 #include "kernels.hpp"
 #include "launch.hpp"
 #include "plan.hpp"
+#include "team.hpp"
 
 namespace sfa {
 
@@ -143,6 +144,82 @@ struct SystemT {
     // FP32 copy of the plan for the mixed-precision solve (T = double only)
     std::unique_ptr<SystemT<float>> inner;
 
+    // Systems with sweeps that do not fit one workgroup, up to 262,144 active
+    // rows (the partials' layout of team.hip; there it is still the faster
+    // one): the loop in launches of a team of workgroups, when no other solve
+    // is under way.  One workgroup for every two slices of 64 rows, 64 to 256
+    // of them: with 64 / 128 / 256 the 129^2 system takes 28.9 / 26.2 / 26.4 us
+    // per iteration, 35,937 rows and 10 colours 59 / 52 / 51, H(curl) with
+    // 102,024 rows 68 / 52 / 43, 274,625 rows 140 / 99 / 88.  Plain and Jacobi
+    // CG stay with their two launches: 2D, 14,400 rows, 11.4 us against 14.3.
+    TeamArgs<T> team{};
+    int team_blocks = 0;     // 0: never
+    bool team_off = false;   // a launch gave up: from now on the launches of an iteration
+    TeamGroup* team_groups = nullptr;
+    static constexpr int kTeamIters = 256;  // most iterations of one such launch: some 20 ms
+    bool in_team() const
+    {
+        return team_blocks > 0 && !team_off && spmv_lanes == 1 && !prof && !launches && !in_block();
+    }
+
+    void create_team()
+    {
+        if (!sweeps || eisen || block.lds > 0 || full.nslices < 1 || full.nslices > 4 * kSpmvMaxBlocks) return;
+        if (std::min(lower.ngroups(), upper.ngroups()) < 1 ||
+            std::max(lower.ngroups(), upper.ngroups()) > kTeamMaxGroups)
+            return;
+        int cus = 0;
+        SFA_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+        int blocks = 64;
+        while (2 * blocks < full.nslices && blocks < kTeamMaxBlocks) blocks *= 2;
+        if (blocks > cus) return;
+        team.full = full.view();
+        std::vector<TeamGroup> g;
+        team.same_wave = 1;
+        team.lower = lower.view();
+        team.upper = upper.view();
+        team.gl = lower.ngroups();
+        team.gu = upper.ngroups();
+        team.fuse = fuse_first_backward ? 1 : 0;
+        for (int i = 0; i < team.gl; i++) g.push_back({sweep_group(lower, i), i, 0});
+        for (int i = 0; i < team.gu; i++) g.push_back({sweep_group(upper, i), i, 0});
+        for (int i = 0; i < team.gl; i++) {
+            if (lower.nrows_of(i) == 0) continue;
+            const int u = upper_of(i);
+            if (u < 0) team.same_wave = 0;
+            else g[team.gl + u].turn = i;
+        }
+        team_groups = dev_alloc<TeamGroup>(g.size());
+        SFA_HIP(hipMemcpy(team_groups, g.data(), g.size() * sizeof(TeamGroup), hipMemcpyHostToDevice));
+        for (T** v : {&team.z0, &team.rs}) {
+            if (v == &team.rs && team.same_wave) continue;
+            *v = dev_alloc<T>(n + 1);
+            SFA_HIP(hipMemset(*v, 0, (n + 1) * sizeof(T)));
+        }
+        team.sync = dev_alloc<unsigned>(kTeamSyncWords);
+        team.groups = team_groups;
+        team.full_slices = full.nslices;
+        team.full_row0 = full.row0(0);
+        team.n = n;
+        team.n_active = n_active;
+        team.x = x;
+        team.r = r;
+        team.d = d;
+        team.d1 = d1;
+        team.z = z;
+        team.m = m;
+        team.q = q;
+        team.diag = diag;
+        team.omega = w();
+        team.c2 = c2();
+        team.st = state;
+        team.ps = ps;
+        team.pb = pb;
+        team.grp = grp;
+        team.max_iters = kTeamIters;
+        team_blocks = blocks;
+    }
+
     // Launches fn(); in a profiled solve, between two events on stream s.
     template <class Fn>
     void run(hipStream_t s, int klass, double bytes, Fn&& fn)
@@ -180,11 +257,15 @@ struct SystemT {
         shares_perm = false;
         for (void* p : {(void*)diag, (void*)x, (void*)r, (void*)b, (void*)d, (void*)d1,
                         (void*)z, (void*)q, (void*)m, (void*)io, (void*)io2, (void*)io3,
-                        (void*)dkeep, (void*)state, (void*)hist, (void*)ps, (void*)pu, (void*)pb, (void*)grp})
+                        (void*)dkeep, (void*)team.z0, (void*)team.rs, (void*)team.sync,
+                        (void*)team_groups, (void*)state, (void*)hist, (void*)ps, (void*)pu, (void*)pb, (void*)grp})
             dev_free(p);
         perm = nullptr;
         diag = x = r = b = d = d1 = z = q = m = io = io2 = io3 = dkeep = nullptr;
         hist = ps = pu = pb = grp = nullptr;
+        team = TeamArgs<T>{};
+        team_groups = nullptr;
+        team_blocks = 0;
         state = nullptr;
         pinned_free(host_state);
         host_state = nullptr;
@@ -342,6 +423,7 @@ struct SystemT {
         init.maxK = n;
         SFA_HIP(hipMemcpy(state, &init, sizeof(SolveState), hipMemcpyHostToDevice));
         host_state = pinned_alloc<SolveState>(1);
+        create_team();
     }
 
     // ---------------------------------------------------------------- phases
@@ -814,20 +896,42 @@ struct SystemT {
     void solve(T* ux, const T* ub, T* ures, double precision, int print_modulo,
                int device_pointers, sfa_solve_info* info)
     {
+        SolveGuard guard(device);
         hipStream_t s = begin_solve(ux, ub, ures, precision, print_modulo, device_pointers);
-        iterate(s);
+        if (!iterate(s)) {  // given up: once more, by the launches of an iteration
+            s = begin_solve(ux, ub, ures, precision, print_modulo, device_pointers);
+            iterate(s);
+        }
         finish_solve(s, ux, ures, print_modulo, device_pointers, info);
     }
 
-    // Runs iterations until the state says the loop has ended.
-    void iterate(hipStream_t s)
+    // Runs iterations until the state says the loop has ended.  False: a
+    // team's launch gave up, and the solve is to be started again (team_off
+    // is then set).
+    bool iterate(hipStream_t s)
     {
         while (in_block() && !host_state->done) {
             SFA_HIP(launch_block_solve<T>(s, block.M, block.lds, state, x, r, b, d, d1, 0, kBlockIters,
                                           0., 0., 0, (const T*)nullptr));
             read_state();
         }
-        if (host_state->done) return;
+        if (host_state->done) return true;
+        while (in_team() && SolveGuard::alone(device) && team_acquire(device, team_blocks)) {
+            try {
+                SFA_HIP(launch_team<T>(s, team, team_blocks));
+                read_state();
+            } catch (...) {
+                (void)hipStreamSynchronize(s);
+                team_release(device, team_blocks);
+                throw;
+            }
+            team_release(device, team_blocks);
+            if (host_state->team_lost) {
+                team_off = true;
+                return false;
+            }
+            if (host_state->done) return true;
+        }
         // Iterations: replay a captured chunk, predicting from the z.r history
         // how many chunks to queue before the next look at the state.
         const int G = 4;
@@ -839,6 +943,7 @@ struct SystemT {
             if (host_state->done) break;
             queued = predict_chunks(G);
         }
+        return true;
     }
 
     // The same solve, every kernel launched on its own between two events.
@@ -1035,6 +1140,7 @@ struct SystemT {
         if (!(rtol > 0) || !(inner_rtol > 0) || !(inner_rtol < 1) || max_outer < 0)
             throw Error{SFA_ERR_INVALID, "need rtol > 0, 0 < inner_rtol < 1, max_outer >= 0"};
         SFA_HIP(hipSetDevice(device));
+        SolveGuard guard(device);
         hipStream_t s = stream;
         inner->stream = s;
         const T* src_x = ux;
@@ -1083,20 +1189,30 @@ struct SystemT {
                 SFA_HIP(hipMemcpyAsync(inner->dkeep, dlast, n * sizeof(float),
                                        hipMemcpyDeviceToDevice, s));
             }
-            inner->start(s, 1.0, -3, 0., 0, inner_rtol * inner_rtol, nullptr, zr_prev, zr_end, k_end);
-            // Continue only where the FP64 residual agrees with the recursive
-            // one the last inner solve ended with: a drifted FP32 residual
-            // makes the old direction unfit (beta far too large).
-            if (inner->in_block()) {
-                continued += inner->host_state->continued;
-            } else if (zr_prev > 0. && !inner->host_state->done &&
-                       inner->host_state->zr <= kContinueGap * zr_end) {
-                launch_direction_continue(s, inner->state, inner->n_active, inner->d,
-                                          (const float*)inner->dkeep, zr_prev,
-                                          (int)std::min<long long>(inner->n, std::max(100LL, 3LL * k_end)));
-                continued++;
+            const auto inner_solve = [&]() -> bool {
+                inner->start(s, 1.0, -3, 0., 0, inner_rtol * inner_rtol, nullptr, zr_prev, zr_end, k_end);
+                // Continue only where the FP64 residual agrees with the recursive
+                // one the last inner solve ended with: a drifted FP32 residual
+                // makes the old direction unfit (beta far too large).
+                bool cont = false;
+                if (inner->in_block()) {
+                    cont = inner->host_state->continued != 0;
+                } else if (zr_prev > 0. && !inner->host_state->done &&
+                           inner->host_state->zr <= kContinueGap * zr_end) {
+                    launch_direction_continue(s, inner->state, inner->n_active, inner->d,
+                                              (const float*)inner->dkeep, zr_prev,
+                                              (int)std::min<long long>(inner->n, std::max(100LL, 3LL * k_end)));
+                    cont = true;
+                }
+                if (!inner->iterate(s)) return false;
+                continued += cont ? 1 : 0;
+                return true;
+            };
+            if (!inner_solve()) {  // given up: once more, by the launches of an iteration
+                launch_fill(s, inner->x, 0.0f, n);
+                launch_fill(s, inner->r, 0.0f, n);
+                inner_solve();
             }
-            inner->iterate(s);
             const SolveState& ist = *inner->host_state;
             if (ist.exit_reason == SFA_EXIT_BREAKDOWN) break;
             // z.r of the iterate that formed the last direction (the stopping
