@@ -82,10 +82,12 @@ void launch_init_state(hipStream_t s, SolveState* st, const T* b, int n, double 
 // MatrixCSR::apply: dest[row] = sum (scaling*v)*src[col], over a part's rows.
 // (row0, nrows): a group whose rows are row0 .. row0+nrows-1 in slice order;
 // row0 = -1 makes the kernels read row ids from the part's row list.
-// lanes: lanes per row (1, 2, 4, 8); every value gives the same bits.
+// lanes: lanes per row (1, 2, 4, 8); every value gives the same bits.  gw: the
+// part's entries per lane when all its slices have the same number, else -1.
+// src needs no zero slot; dest is not src.
 template <typename T>
 void launch_apply(hipStream_t s, SellViewT<T> A, int nslices, int row0, int nrows, const T* src,
-                  T* dest, T scaling, int lanes = 1);
+                  T* dest, T scaling, int lanes = 1, int gw = -1);
 
 // --- restart (K = 0) ---
 enum ResidualMode { RES_ONLY = 0, RES_PLAIN = 1, RES_JACOBI = 2 };

@@ -1101,18 +1101,29 @@ struct SystemT {
             apply_part.upload(p);
             has_apply_part = true;
         }
-        hipStream_t s = stream;
-        // source with a zero slot at n: use the x-sized buffer m
-        T* srcbuf = q;
+        // Device vectors come from work on the null stream (see
+        // order_after_null_stream): the product itself runs there when the
+        // system has no stream of the caller's, which takes an event and a
+        // wait less per call.  Nothing of an earlier call is still queued on
+        // the system's own stream: every call waits for its work.
+        hipStream_t s = device_pointers && stream == own_stream ? nullptr : stream;
+        // host vectors, and a dest that overlaps src, go through a copy of src
+        const T* from = src;
+        T* out = dest;
         if (device_pointers) {
-            order_after_null_stream(s);
-            SFA_HIP(hipMemcpyAsync(srcbuf, src, n * sizeof(T), hipMemcpyDeviceToDevice, s));
-        } else
-            SFA_HIP(hipMemcpyAsync(srcbuf, src, n * sizeof(T), hipMemcpyHostToDevice, s));
-        launch_fill(s, srcbuf + n, T(0), 1);
-        T* out = device_pointers ? dest : io;
+            const char *d0 = reinterpret_cast<const char*>(dest), *s0 = reinterpret_cast<const char*>(src);
+            const std::ptrdiff_t size = (std::ptrdiff_t)n * (std::ptrdiff_t)sizeof(T);
+            if (d0 < s0 + size && s0 < d0 + size) {
+                SFA_HIP(hipMemcpyAsync(io2, src, n * sizeof(T), hipMemcpyDeviceToDevice, s));
+                from = io2;
+            }
+        } else {
+            SFA_HIP(hipMemcpyAsync(io2, src, n * sizeof(T), hipMemcpyHostToDevice, s));
+            from = io2;
+            out = io;
+        }
         launch_apply(s, apply_part.view(), apply_part.nslices, apply_part.row0(0), apply_part.nrows_of(0),
-                     srcbuf, out, T(scaling), spmv_lanes);
+                     from, out, T(scaling), spmv_lanes, apply_part.width(0));
         if (!device_pointers)
             SFA_HIP(hipMemcpyAsync(dest, io, n * sizeof(T), hipMemcpyDeviceToHost, s));
         SFA_HIP(hipStreamSynchronize(s));
