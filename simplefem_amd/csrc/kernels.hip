@@ -37,6 +37,13 @@ int spmv_blocks(int nslices)
     return b < 1 ? 1 : (b > kSpmvMaxBlocks ? kSpmvMaxBlocks : b);
 }
 
+int spmv_split_blocks(int nslices)
+{
+    const int b = (nslices + kSpmvWaves - 1) / kSpmvWaves;
+    const int rounds = (b + kSpmvSplitMaxBlocks - 1) / kSpmvSplitMaxBlocks;
+    return b < 1 ? 1 : (b + rounds - 1) / rounds;  // the last round as full as the others
+}
+
 int vec_reduce_blocks(int n)
 {
     const int b = (n + dev::kVecBlock - 1) / dev::kVecBlock;
@@ -994,6 +1001,94 @@ __global__ void __launch_bounds__(kSpmvBlock) k_spmv_dir(SellViewT<T> A, int nsl
     block_partial<kSpmvBlock>(part_sum, &spart[blockIdx.x]);
 }
 
+// The direction of k_spmv_dir alone: opens the iteration and stores
+// dn = src + beta*dold (rows past n_active keep theirs in both buffers).
+template <typename T>
+__global__ void __launch_bounds__(kVecBlock) k_direction(int n_active, SolveState* st, int p,
+                                                         const T* src, const T* dold, T* dnew,
+                                                         const double* fpart, int nfold,
+                                                         const double* fpartb, int nfoldb,
+                                                         const double* gsum, int ngroups)
+{
+    constexpr int B = 8;  // rows in flight per thread, the first of them ahead of the state
+    const int stride = gridDim.x * kVecBlock;
+    int i0 = xcd_block(blockIdx.x, gridDim.x) * kVecBlock + threadIdx.x;
+    T ss[B], dd[B];
+    auto load = [&] {
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const int i = i0 + u * stride;
+            ss[u] = i < n_active ? src[i] : T(0);
+            dd[u] = i < n_active ? dold[i] : T(0);
+        }
+    };
+    load();
+    const int fold = st->fold[p];
+    const int Kit = st->Kp[p];
+    const double zr_old = st->zrp[p];
+    if (__syncthreads_or(st->done)) return;  // see k_spmv_dir
+    double zr_new = 0.;
+    if (fold) {
+        __shared__ double sh;
+        if (threadIdx.x < kWave) {
+            double t = 0.;
+            for (int g = 0; g < ngroups; g++) t += gsum[g];
+            t += wave_fold(fpart, nfold);
+            if (fpartb) t += wave_fold(fpartb, nfoldb);
+            if (threadIdx.x == 0) sh = t;
+        }
+        __syncthreads();
+        zr_new = sh;
+    }
+    double beta_d;
+    if (open_step(st, p, fold, zr_old, Kit, zr_new, &beta_d)) return;
+    const T beta = (T)beta_d;
+    for (;;) {
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const int i = i0 + u * stride;
+            if (i < n_active) dnew[i] = fold ? ss[u] + beta * dd[u] : dd[u];
+        }
+        if (n_active - i0 <= B * stride) return;  // i0 stays below n_active
+        i0 += B * stride;
+        load();
+    }
+}
+
+// q = A d and the d.Ad partials of k_spmv_dir, d stored by k_direction: one
+// gather per entry where k_spmv_dir has two, which bound it, and so few
+// registers (8 entries loaded ahead; 16: 75 us
+// per iteration of the first system below, 8: 66) that 2,048 blocks are
+// resident (4,096: 67 us).  us per iteration of plain CG,
+// k_spmv_dir -> both kernels: 795,024 H(curl) rows, 12.8 M entries 96 -> 63,
+// 338,364 rows, 5.4 M entries 58 -> 37, 912,673 rows, 13.5 M entries 70 -> 57,
+// 274,625 rows, 4.0 M entries 36 -> 31; of Rainbow CG-SSOR on the first 144 -> 128.
+template <typename T>
+__global__ void __launch_bounds__(kSpmvBlock) k_spmv(SellViewT<T> A, int nslices, int row0,
+                                                     int nrows, const SolveState* st,
+                                                     const T* d, T* q, double* spart, int gw)
+{
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int stride = gridDim.x * kSpmvWaves;
+    const bool done = st->done;  // no block of this launch sets it
+    double part = 0.;
+    for (int slice = xcd_block(blockIdx.x, gridDim.x) * kSpmvWaves + wave; slice < nslices; slice += stride) {
+        SellChunk<T, 8> R;
+        sell_prefetch(A, slice, slice, 0, gw, lane, R);
+        const int row = group_row_at(A, slice, slice, lane, row0, nrows);
+        const T dr = d[row >= 0 ? row : A.zero];
+        if (done) return;
+        const T acc = sell_finish<false>(A, R, [&](unsigned c) { return d[c]; }, T(0));
+        if (row >= 0) {
+            q[row] = acc;
+            part += (double)(dr * acc);
+        }
+    }
+    if (done) return;
+    block_partial<kSpmvBlock>(part, &spart[blockIdx.x]);
+}
+
 // d.Ad step from dpart, then x += a dx; r -= a q; z.r by mode
 // (solver/sparsesolver.cpp:160-174, 372-389, 952-968) into zpart.
 template <typename T>
@@ -1287,6 +1382,19 @@ void launch_spmv_dir(hipStream_t s, SellViewT<T> A, int nslices, int row0, int n
 }
 
 template <typename T>
+void launch_direction_spmv(hipStream_t s, SellViewT<T> A, int nslices, int row0, int nrows,
+                           int n_active, SolveState* st, int p, const T* src, const T* dold, T* dnew,
+                           T* q, double* spmv_partials, const double* fold_partials, int nfold,
+                           const double* fold_partials_b, int nfold_b, const double* group_sums,
+                           int ngroups, int gw)
+{
+    launch(k_direction<T>, dim3(vec_reduce_blocks(n_active)), dim3(kVecBlock), s, n_active, st, p,
+           src, dold, dnew, fold_partials, nfold, fold_partials_b, nfold_b, group_sums, ngroups);
+    launch(k_spmv<T>, dim3(spmv_split_blocks(nslices)), dim3(kSpmvBlock), s, A, nslices, row0,
+           nrows, (const SolveState*)st, (const T*)dnew, q, spmv_partials, gw);
+}
+
+template <typename T>
 void launch_update(hipStream_t s, UpdateMode mode, SolveState* st, int p, int n_active, T* x,
                    T* r, const T* dx, const T* q, T* z, const T* diag_or_precon, T omega,
                    const double* dad_partials, int ndad, double* zr_partials)
@@ -1353,6 +1461,10 @@ void launch_add_correction(hipStream_t s, double* x, const float* e, int n)
     template void launch_eisenstat_upper<T>(hipStream_t, SellViewT<T>, int, int, int, int,     \
                                             SolveState*, int, int, const T*, const T*, T*, T*, \
                                             const T*, T, const double*, int, int, int);        \
+    template void launch_direction_spmv<T>(hipStream_t, SellViewT<T>, int, int, int, int,      \
+                                           SolveState*, int, const T*, const T*, T*, T*,       \
+                                           double*, const double*, int, const double*, int,    \
+                                           const double*, int, int);                           \
     template void launch_spmv_dir<T>(hipStream_t, SellViewT<T>, int, int, int, int,            \
                                      SolveState*, int, const T*, const T*, T*, T*, double*,    \
                                      const double*, int, const double*, int, const double*,    \

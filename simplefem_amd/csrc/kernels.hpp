@@ -64,7 +64,9 @@ constexpr int kSpmvWaves = 4;          // slices per block of the SpMV kernel
 constexpr int kSpmvMaxBlocks = 1024;
 constexpr int kVecReduceBlocks = 512;  // vector kernels with a reduction
 
+constexpr int kSpmvSplitMaxBlocks = 2048;  // k_spmv, see there
 int spmv_blocks(int nslices);
+int spmv_split_blocks(int nslices);
 int vec_reduce_blocks(int n);
 
 // Vector kernels
@@ -212,6 +214,14 @@ void launch_spmv_dir(hipStream_t s, SellViewT<T> A, int nslices, int row0, int n
                      T* q, double* spmv_partials, const double* fold_partials, int nfold,
                      const double* fold_partials_b, int nfold_b, const double* group_sums,
                      int ngroups, int gw, int lanes);
+// The same in two launches, one lane per row: dnew first, then q and the
+// partials (spmv_split_blocks(nslices) of them) from it.
+template <typename T>
+void launch_direction_spmv(hipStream_t s, SellViewT<T> A, int nslices, int row0, int nrows,
+                           int n_active, SolveState* st, int p, const T* src, const T* dold, T* dnew,
+                           T* q, double* spmv_partials, const double* fold_partials, int nfold,
+                           const double* fold_partials_b, int nfold_b, const double* group_sums,
+                           int ngroups, int gw);
 enum UpdateMode { UPD_PLAIN = 0, UPD_JACOBI = 1, UPD_EISENSTAT = 2 };
 // Forms d.Ad from dad_partials (ndad), breakdown tests, alpha; then
 // x += a*dx; r -= a*q; z.r per mode into zr_partials (one per block).

@@ -162,9 +162,27 @@ struct SystemT {
         return team_blocks > 0 && !team_off && spmv_lanes == 1 && !prof && !launches && !in_block();
     }
 
+    // Whether the direction is stored by a kernel of its own: where one kernel
+    // for both, which fills the chip with kSpmvMaxBlocks blocks, needs a second
+    // round of slices.  Up to there a launch more costs more than it saves
+    // (plain CG, us per iteration, one kernel -> two: 117,649 rows 18 -> 23,
+    // 160,804 rows 25 -> 28), beyond it less (274,625 rows 36 -> 31; see k_spmv).
+    bool spmv_split(int lanes) const { return lanes == 1 && full.nslices > kSpmvWaves * kSpmvMaxBlocks; }
+    int spmv_partials() const
+    {
+        return spmv_split(spmv_lanes) ? spmv_split_blocks(full.nslices) : spmv_blocks(full.nslices * spmv_lanes);
+    }
+    // An iteration's direction and product over P's rows (launch_spmv_dir).
+    template <class... Args>
+    void direction_product(int lanes, Args... args)
+    {
+        if (spmv_split(lanes)) launch_direction_spmv(args...);
+        else launch_spmv_dir(args..., lanes);
+    }
+
     void create_team()
     {
-        if (!sweeps || eisen || block.lds > 0 || full.nslices < 1 || full.nslices > 4 * kSpmvMaxBlocks) return;
+        if (!sweeps || eisen || block.lds > 0 || full.nslices < 1 || full.nslices > kSpmvWaves * kSpmvMaxBlocks) return;
         if (std::min(lower.ngroups(), upper.ngroups()) < 1 ||
             std::max(lower.ngroups(), upper.ngroups()) > kTeamMaxGroups)
             return;
@@ -412,7 +430,7 @@ struct SystemT {
         io3 = dev_alloc<T>(n);
         state = dev_alloc<SolveState>(1);
         hist = dev_alloc<double>((size_t)n + 1);
-        ps = dev_alloc<double>(std::max(kSpmvMaxBlocks, kVecReduceBlocks));
+        ps = dev_alloc<double>(std::max({kSpmvMaxBlocks, kSpmvSplitMaxBlocks, kVecReduceBlocks}));
         pu = dev_alloc<double>(std::max({full.nslices, kVecReduceBlocks, 1}));
         pb = dev_alloc<double>(std::max(sweeps ? upper.nslices : 0, 1));
         int ngr = 1;
@@ -521,7 +539,7 @@ struct SystemT {
     // schedule; dd: the iteration's direction.
     void forward_iteration(hipStream_t s, int p, const T* dd)
     {
-        const int nspmv = spmv_blocks(full.nslices * spmv_lanes);
+        const int nspmv = spmv_partials();
         const int G = lower.ngroups();
         const int g0 = merge_first_forward ? 1 : 0;
         for (const SweepLaunch& e : fwd_sched) {
@@ -600,7 +618,7 @@ struct SystemT {
         // vector streams per row: x r/w, d, r r/w, q, diag, m (iteration);
         // r, diag, m (restart); + z when fused
         const double per_row = mode == FWD_RESTART ? 24.0 : 64.0;
-        const int nspmv = spmv_blocks(full.nslices * spmv_lanes);
+        const int nspmv = spmv_partials();
         const int G = L.ngroups();
         const int g0 = merge_first_forward ? 1 : 0;
         for (int g = g0; g < G; g++) {
@@ -703,17 +721,17 @@ struct SystemT {
         T* dold = p ? d1 : d;
         T* dnew = p ? d : d1;
         const double spmv_bytes = full.bytes_all(32.0);  // src, dold, dnew, q
-        const int nspmv = spmv_blocks(full.nslices * spmv_lanes);
+        const int nspmv = spmv_partials();
         const int nvec = vec_reduce_blocks(n_active);
         switch (method) {
         case SFA_METHOD_CG:
         case SFA_METHOD_DIAGONAL: {
             const bool jac = method == SFA_METHOD_DIAGONAL;
             run(s, SFA_KERNEL_SPMV, spmv_bytes, [&] {
-                launch_spmv_dir(s, F, full.nslices, full.row0(0), full.nrows_of(0), n_active,
+                direction_product(spmv_lanes, s, F, full.nslices, full.row0(0), full.nrows_of(0), n_active,
                                 state, p, jac ? z : r, dold, dnew, q, ps, pu, nvec,
                                 (const double*)nullptr, 0, (const double*)nullptr, 0,
-                                full.width(0), spmv_lanes);
+                                full.width(0));
             });
             run(s, SFA_KERNEL_UPDATE, (jac ? 64.0 : 48.0) * na, [&] {
                 launch_update(s, jac ? UPD_JACOBI : UPD_PLAIN, state, p, n_active, x, r, dnew, q,
@@ -730,13 +748,13 @@ struct SystemT {
             const int nt = (int)spmv_tail.size();
             const int ta = nt > 0 ? spmv_tail[0] : -1, tb = nt > 1 ? spmv_tail[1] : -1;
             run(s, SFA_KERNEL_SPMV, spmv_bytes, [&] {
-                launch_spmv_dir(s, F, full.nslices, full.row0(0), full.nrows_of(0), n_active,
+                direction_product(spmv_lanes, s, F, full.nslices, full.row0(0), full.nrows_of(0), n_active,
                                 state, p, z, dold, dnew, q, ps,
                                 ta >= 0 ? pb + upper.group_begin(ta) : pb,
                                 ta >= 0 ? upper.group_count(ta) : 0,
                                 tb >= 0 ? pb + upper.group_begin(tb) : (const double*)nullptr,
                                 tb >= 0 ? upper.group_count(tb) : 0, grp, G - nt,
-                                full.width(0), spmv_lanes);
+                                full.width(0));
             });
             forward_iteration(s, p, dnew);
             backward_iteration(s, dnew);
@@ -763,11 +781,12 @@ struct SystemT {
 
     int kernels_per_iteration() const
     {
+        const int split = spmv_split(spmv_lanes) ? 1 : 0;
         switch (method) {
         case SFA_METHOD_CG:
-        case SFA_METHOD_DIAGONAL: return 2;
+        case SFA_METHOD_DIAGONAL: return 2 + split;
         case SFA_METHOD_SSOR:
-        case SFA_METHOD_RAINBOW: return 1 + (int)fwd_sched.size() + (int)bwd_sched.size();
+        case SFA_METHOD_RAINBOW: return 1 + split + (int)fwd_sched.size() + (int)bwd_sched.size();
         default: return 2 + lower.ngroups() + upper.ngroups();
         }
     }
@@ -1296,7 +1315,7 @@ struct SystemT {
         SolveState* ts = dev_alloc<SolveState>(1);
         double* th = dev_alloc<double>(2);
         double* tz = dev_alloc<double>(nscratch);  // zero partials to fold
-        double* tp = dev_alloc<double>(kSpmvMaxBlocks);
+        double* tp = dev_alloc<double>(std::max(kSpmvMaxBlocks, kSpmvSplitMaxBlocks));
         hipEvent_t e0 = nullptr, e1 = nullptr;
         auto cleanup = [&] {
             if (e0) (void)hipEventDestroy(e0);
@@ -1316,9 +1335,9 @@ struct SystemT {
             SFA_HIP(hipEventCreate(&e1));
             const SellViewT<T> F = full.view();
             auto once = [&](int lanes) {
-                launch_spmv_dir(stream, F, full.nslices, full.row0(0), full.nrows_of(0), n_active,
+                direction_product(lanes, stream, F, full.nslices, full.row0(0), full.nrows_of(0), n_active,
                                 ts, 0, z, d, d1, q, tp, tz, nfold, (const double*)nullptr, 0,
-                                tz, ngroups, full.width(0), lanes);
+                                tz, ngroups, full.width(0));
             };
             const int cand[SFA_SPMV_MAPPINGS] = {1, 2, 4, 8};
             const int main = full.main_bucket();
